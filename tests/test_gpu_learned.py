@@ -474,3 +474,34 @@ def test_network_tiles(pkg, orc, ref, gpu_lib, n, sub):
             L, g, _ = ref.loss_and_grad(params.astype(np.float64), f, rows_t, tgt, w)
             assert res.loss == pytest.approx(L, rel=1e-5)
             assert np.linalg.norm(grad - g) <= 1e-5 * np.linalg.norm(g)
+
+
+def _cluster(orc, n, seed=3):
+    """n particles, each within h of every other."""
+    rng = np.random.default_rng(seed)
+    p = orc.particles(n)
+    p["pos"][:, :3] = rng.uniform(0.0, 0.008, (n, 3)).astype(np.float32)
+    p["vel"][:, :3] = rng.normal(0, 5, (n, 3)).astype(np.float32)
+    return p
+
+
+def test_messages_16bit_keep_first_layer_weights(pkg, orc, ref, gpu_lib):
+    """First-layer weights that BF16 would all round towards zero, by 0.49 units in its
+    last place: rounded so, the messages are 2.7e-3 off; what rounds at random (inputs,
+    activations, W2) averages out over 129 pairs and 64 units to 5e-4."""
+    n = 130
+    params = ref.init_params(29)
+    params[ref.NPARAMS - 195:] += np.random.default_rng(n).normal(0, 0.05, 195).astype(np.float32)
+    w1 = params[:576]
+    w1[:] = (w1.view(np.uint32) & 0xffff0000).view(np.float32)
+    w1 += np.sign(w1) * np.float32(0.49) * np.exp2(np.floor(np.log2(np.abs(w1))) - 7).astype(np.float32)
+    with pkg.Simulation(n) as sim:
+        sim.upload(_cluster(orc, n))
+        sim.rho_pres()
+        norm = _norm(pkg)
+        norm.rho_scale = float(1.3 / sim.download()["extras"][:, 0].mean())
+        norm.pi_scale = float(1.0 / sim.download()["extras"][:, 1].mean()) * float(sim.download()["extras"][:, 0].mean())
+        sim.mlp_set(params, norm)
+        half = sim.mlp_predict(path=1).astype(np.float64)
+        full = sim.mlp_predict(path=0).astype(np.float64)
+    assert np.linalg.norm(half - full) <= 1.2e-3 * np.linalg.norm(full)
