@@ -505,3 +505,49 @@ def test_messages_16bit_keep_first_layer_weights(pkg, orc, ref, gpu_lib):
         half = sim.mlp_predict(path=1).astype(np.float64)
         full = sim.mlp_predict(path=0).astype(np.float64)
     assert np.linalg.norm(half - full) <= 1.2e-3 * np.linalg.norm(full)
+
+
+@pytest.mark.parametrize("z1", [-4.0, -60.0, -3e4, 1e5, 0.5])
+@pytest.mark.parametrize("z2", [-5.0, -100.0, -2e4, 3.5, 700.0])
+def test_messages_16bit_gelu_tails(pkg, orc, ref, gpu_lib, z1, z2):
+    """16-bit messages where every activation of a layer has the same input, in
+    the tails of the GELU: the training form stays at -0.00197 below -3, and an
+    offset there has one sign over all pairs.  Bounds of an activation's error:
+    1e-5 in the negative tail (coefficients and FP16 rounding), elsewhere the
+    lookup's 2^-7 of the value; inputs beyond 65504 saturate.  The second layer
+    passes the first's error on."""
+    n = 34
+    params = np.zeros(ref.NPARAMS, np.float32)
+    params[576:640] = z1
+    params[640:640 + 4096] = np.eye(64, dtype=np.float32).ravel()
+    params[4736:4800] = z2
+    params[4800:4992] = 1.0
+    h1 = ref.gelu(min(z1, 65504.0))
+    h2 = ref.gelu(min(h1 + z2, 65504.0))
+    err1 = 1e-5 if z1 < -3 else abs(h1) * 2.0**-7
+    err2 = 1e-5 if h1 + z2 < -3 else abs(h2) * 2.0**-7
+    with pkg.Simulation(n) as sim:
+        sim.upload(_cluster(orc, n))
+        sim.mlp_set(params, _norm(pkg))
+        got = sim.mlp_predict(path=1).astype(np.float64)
+    slope = 1.0 if h1 + err1 + z2 > -3 else 0.0
+    assert np.abs(got / (64 * (n - 1)) - h2).max() <= err2 + slope * err1
+
+
+def test_messages_16bit_infinite_activations(pkg, orc, ref, gpu_lib):
+    """A first layer that overflows to minus infinity ends in the GELU's
+    negative tail, as any large negative input does."""
+    n = 34
+    params = np.zeros(ref.NPARAMS, np.float32)
+    params[6 * 64:7 * 64] = params[576:640] = -3e38
+    params[4800:4992] = 1.0
+    params[640:640 + 4096] = np.eye(64, dtype=np.float32).ravel()
+    params[4736:4800] = -5.0
+    with pkg.Simulation(n) as sim:
+        sim.upload(_cluster(orc, n))
+        sim.rho_pres()
+        norm = _norm(pkg)
+        norm.rho_scale = float(16.0 / sim.download()["extras"][:, 0].min())
+        sim.mlp_set(params, norm)
+        got = sim.mlp_predict(path=1).astype(np.float64)
+    assert np.abs(got / (64 * (n - 1)) - ref.gelu(-5.0)).max() <= 1e-5
