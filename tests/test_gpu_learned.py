@@ -551,3 +551,20 @@ def test_messages_16bit_infinite_activations(pkg, orc, ref, gpu_lib):
         sim.mlp_set(params, norm)
         got = sim.mlp_predict(path=1).astype(np.float64)
     assert np.abs(got / (64 * (n - 1)) - ref.gelu(-5.0)).max() <= 1e-5
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("n", [2, 34, 300])
+def test_messages_16bit_show_nonfinite_inputs(pkg, orc, ref, gpu_lib, value, n):
+    """A particle of non-finite velocity makes its own message and its
+    neighbours' non-finite, and no other's: two clusters, one of them with it."""
+    p = np.concatenate([_cluster(orc, n), _cluster(orc, n, 4)])
+    p["pos"][n:, 0] += 0.1
+    p["vel"][n // 2, 1] = value
+    with pkg.Simulation(2 * n) as sim:
+        sim.upload(p)
+        sim.mlp_set(ref.init_params(31), _norm(pkg))
+        half = sim.mlp_predict(path=1)
+        full = sim.mlp_predict(path=0)
+    assert not np.isfinite(half[:n]).any() and np.isfinite(half[n:]).all()
+    assert np.array_equal(np.isfinite(half), np.isfinite(full))
