@@ -568,3 +568,34 @@ def test_messages_16bit_show_nonfinite_inputs(pkg, orc, ref, gpu_lib, value, n):
         full = sim.mlp_predict(path=0)
     assert not np.isfinite(half[:n]).any() and np.isfinite(half[n:]).all()
     assert np.array_equal(np.isfinite(half), np.isfinite(full))
+
+
+@pytest.mark.parametrize("layer", ["W2", "W3"])
+def test_messages_16bit_show_diverged_weights(pkg, orc, ref, gpu_lib, layer):
+    """Weights that an Adam update made NaN (eps = 0 and no gradient: 0/0) in
+    one layer alone make the messages NaN on both paths.  A unit whose input
+    weights are zero passes 0 on, so its output weights get no gradient."""
+    n = 34
+    d = ref.unpack(ref.init_params(31))
+    d["w3"] += np.random.default_rng(32).normal(0, 0.05, d["w3"].shape)
+    if layer == "W2":
+        d["w1"][:, 5] = 0.0
+    else:
+        d["w2"][:, 5] = 0.0
+    p = _cluster(orc, n)
+    q = _cluster(orc, n)
+    q["vel"][:, :3] += np.random.default_rng(33).normal(0, 5, (n, 3)).astype(np.float32)
+    with pkg.Simulation(n) as sim, pkg.Simulation(n) as later:
+        sim.upload(p)
+        later.upload(q)
+        sim.mlp_set(ref.pack(d).astype(np.float32), _norm(pkg))
+        sim.mlp_train(later, lr=1e-3, eps=0.0)
+        got = ref.unpack(sim.mlp_get()[0])
+        for name in ("w1", "b1", "w2", "b2", "w3", "b3"):
+            bad = np.isnan(got[name])
+            if name == layer.lower():
+                assert bad[5].all() and not np.delete(bad, 5, axis=0).any()
+            else:
+                assert not bad.any()
+        assert np.isnan(sim.mlp_predict(path=1)).all()
+        assert np.isnan(sim.mlp_predict(path=0)).all()
