@@ -91,7 +91,7 @@ struct MlpWork {
 };
 
 constexpr int kMlpPackA = 4 * 64 * 8 + 4 * 2 * 64 * 8 + 2 * 64 * 8;  // 16-bit entries
-constexpr int kMlpPackC = kMlpHidden + 8;                            // float entries
+constexpr int kMlpPackC = 2 * kMlpHidden + 8;                        // float entries
 // Totals of a training step: loss sum, pairs, targets of weight 1.
 constexpr size_t kTrainSumsBytes = 24;
 constexpr uint32_t kMaxTrainWaves = 4u * 2048u;

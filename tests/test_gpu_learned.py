@@ -599,3 +599,53 @@ def test_messages_16bit_show_diverged_weights(pkg, orc, ref, gpu_lib, layer):
                 assert not bad.any()
         assert np.isnan(sim.mlp_predict(path=1)).all()
         assert np.isnan(sim.mlp_predict(path=0)).all()
+
+
+@pytest.mark.parametrize("case", ["plain", "small", "tiny", "huge", "units", "low edge", "high edge", "outputs"])
+def test_messages_16bit_any_weight_size(pkg, orc, ref, gpu_lib, case):
+    """W2 and W3 of any size, beyond FP16's range and among its subnormals, in
+    networks whose activations are of ordinary size: the earlier layer or the
+    later one is scaled the other way.  W2 has one scale a unit where a unit's
+    largest (halved) weight leaves [2^-8, 65504], none inside it.  Bound: one
+    rounding of each input to BF16, 2^-9; over 64 units and 129 pairs roundings
+    average out to less."""
+    n = 130
+    rng = np.random.default_rng(41)
+    d = ref.unpack(ref.init_params(29))
+    d["w3"] += rng.normal(0, 0.05, d["w3"].shape)
+    d["b1"], d["b2"] = rng.normal(0, 0.1, 64), rng.normal(0, 0.1, 64)
+    one, two = {"small": (1e4, 1e-4), "tiny": (1e4, 1e-5), "huge": (1e-3, 1e7)}.get(case, (1.0, 1.0))
+    d["w1"] *= one
+    d["b1"] *= one
+    d["w2"] *= two
+    d["b2"] *= min(two * one, 1.0)
+    big = np.abs(d["w2"]).max(axis=0)
+    if case == "units":
+        k = 10.0 ** np.linspace(-3, 3, 64)
+        d["w2"] *= k
+        d["b2"] *= k
+        d["w3"] /= k[:, None]
+    elif case == "low edge":  # half the units one rounding above the edge, half below
+        k = 2.0**-7 / big * np.where(np.arange(64) % 2, 1.001, 0.999)
+        d["w1"] *= 30.0
+        d["b1"] *= 30.0
+        d["w2"] *= k
+    elif case == "high edge":
+        k = 2.0 * 65504 / big * np.where(np.arange(64) % 2, 1.001, 0.999)
+        d["w1"] *= 1e-4
+        d["b1"] *= 1e-4
+        d["w2"] *= k
+    elif case == "outputs":
+        d["w3"] *= [1e-12, 1.0, 1e9]
+    params = ref.pack(d).astype(np.float32)
+    with pkg.Simulation(n) as sim:
+        sim.upload(_cluster(orc, n))
+        sim.rho_pres()
+        norm = _norm(pkg)
+        norm.rho_scale = float(1.3 / sim.download()["extras"][:, 0].mean())
+        norm.pi_scale = float((sim.download()["extras"][:, 0] / sim.download()["extras"][:, 1]).mean())
+        sim.mlp_set(params, norm)
+        half = sim.mlp_predict(path=1).astype(np.float64)
+        full = sim.mlp_predict(path=0).astype(np.float64)
+    assert np.isfinite(full).all()
+    assert (np.linalg.norm(half - full, axis=0) <= 2.0**-9 * np.linalg.norm(full, axis=0)).all()
