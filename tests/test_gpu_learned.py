@@ -606,7 +606,7 @@ def test_messages_16bit_any_weight_size(pkg, orc, ref, gpu_lib, case):
     """W2 and W3 of any size, beyond FP16's range and among its subnormals, in
     networks whose activations are of ordinary size: the earlier layer or the
     later one is scaled the other way.  W2 has one scale a unit where a unit's
-    largest (halved) weight leaves [2^-8, 65504], none inside it.  Bound: one
+    largest weight (half of it for 2 units in 4) leaves [2^-8, 65504], none inside it.  Bound: one
     rounding of each input to BF16, 2^-9; over 64 units and 129 pairs roundings
     average out to less."""
     n = 130
@@ -625,13 +625,13 @@ def test_messages_16bit_any_weight_size(pkg, orc, ref, gpu_lib, case):
         d["w2"] *= k
         d["b2"] *= k
         d["w3"] /= k[:, None]
-    elif case == "low edge":  # half the units one rounding above the edge, half below
-        k = 2.0**-7 / big * np.where(np.arange(64) % 2, 1.001, 0.999)
+    elif case == "low edge":  # half the units just above the edge, half below
+        k = np.where(np.arange(64) % 4 < 2, 2.0**-7, 2.0**-8) / big * np.where(np.arange(64) % 2, 1.001, 0.999)
         d["w1"] *= 30.0
         d["b1"] *= 30.0
         d["w2"] *= k
     elif case == "high edge":
-        k = 2.0 * 65504 / big * np.where(np.arange(64) % 2, 1.001, 0.999)
+        k = np.where(np.arange(64) % 4 < 2, 131008.0, 65504.0) / big * np.where(np.arange(64) % 2, 1.001, 0.999)
         d["w1"] *= 1e-4
         d["b1"] *= 1e-4
         d["w2"] *= k
@@ -649,3 +649,27 @@ def test_messages_16bit_any_weight_size(pkg, orc, ref, gpu_lib, case):
         full = sim.mlp_predict(path=0).astype(np.float64)
     assert np.isfinite(full).all()
     assert (np.linalg.norm(half - full, axis=0) <= 2.0**-9 * np.linalg.norm(full, axis=0)).all()
+
+
+@pytest.mark.parametrize("scale", [3e-6, 2e-5, 6e-5])
+def test_messages_16bit_small_activations(pkg, orc, ref, gpu_lib, scale):
+    """Activations among FP16's subnormals: the lookup takes its values' centres
+    2^-20 apart, so an activation is within 2^-21 and its GELU, of slope 1/2 there, within
+    2^-22 (plus the polynomial's and rounding's 2^-24).  One
+    activation per unit over the range, passed on by a diagonal W3."""
+    n = 34
+    x = np.random.default_rng(43).uniform(-scale, scale, (2, 64))
+    for row in x.astype(np.float32):
+        err = np.zeros(64)
+        for c in range(0, 64, 3):  # three units at a time, one an output
+            params = np.zeros(ref.NPARAMS, np.float32)
+            params[4736:4800] = row
+            for k, u in enumerate(range(c, min(c + 3, 64))):
+                params[4800 + 3 * u + k] = 1.0
+            with pkg.Simulation(n) as sim:
+                sim.upload(_cluster(orc, n))
+                sim.mlp_set(params, _norm(pkg))
+                got = sim.mlp_predict(path=1).astype(np.float64) / (n - 1)
+            for k, u in enumerate(range(c, min(c + 3, 64))):
+                err[u] = np.abs(got[:, k] - ref.gelu(float(row[u]))).max()
+        assert err.max() <= 2.0**-22 + 2.0**-24, err.max()
