@@ -673,3 +673,48 @@ def test_messages_16bit_small_activations(pkg, orc, ref, gpu_lib, scale):
             for k, u in enumerate(range(c, min(c + 3, 64))):
                 err[u] = np.abs(got[:, k] - ref.gelu(float(row[u]))).max()
         assert err.max() <= 2.0**-22 + 2.0**-24, err.max()
+
+
+@pytest.mark.parametrize("n", [64, 65, 66, 129, 256, 257, 321, 513])
+def test_network_long_rows(pkg, orc, ref, gpu_lib, n):
+    """All particles in one grid cell, a stencil row of n slots: rows of more
+    than 64 slots are listed by the whole wave, lists of 256 (16-bit messages,
+    backward pass) and 512 candidates cut them, and a second cluster in the next
+    cell gives a wave a long and a short row.  Messages and gradient against FP64 as in
+    test_network_tiles."""
+    rng = np.random.default_rng(n)
+    params = ref.init_params(29)
+    params[ref.NPARAMS - 195:] += rng.normal(0, 0.05, 195).astype(np.float32)
+    short = 5
+    p = orc.particles(n + short)
+    p["pos"][:, :3] = rng.uniform(0.0001, 0.001, (n + short, 3)).astype(np.float32)
+    p["pos"][n:, 1] += 0.006
+    p["vel"][:, :3] = rng.normal(0, 5, (n + short, 3)).astype(np.float32)
+    q = p.copy()
+    q["vel"][:, :3] += rng.normal(0, 5, (n + short, 3)).astype(np.float32)
+    h = orc.smoothing_length()
+    with pkg.Simulation(n + short) as sim, pkg.Simulation(n + short) as later:
+        sim.upload(p)
+        later.upload(q)
+        sim.mlp_set(params, _norm(pkg))
+        half = sim.mlp_predict(path=1)
+        pred = sim.mlp_predict(path=0)
+        now = sim.download()
+        _, perm = sim.download_grid()
+        slots = np.arange(n + short)
+        rows_t, rows_j, margin = _cpu_pairs(now, perm, h, slots)
+        assert margin > 1e-6
+        f = _features(ref, now, perm, slots, rows_t, rows_j, h)
+        m, _ = ref.forward(params.astype(np.float64), f)
+        want = np.zeros((n + short, 3))
+        np.add.at(want, rows_t, m)
+        assert np.abs(pred[perm] - want).max() <= 6e-8 * n * n + 1e-6 * np.abs(m).max() * n
+        # 16-bit: all pairs are nearly alike, so the lookups' errors (2^-7 of a value) do not average over them.
+        assert np.linalg.norm(half[perm] - want) <= 2.0**-7 * np.linalg.norm(want)
+        res, grad = sim.mlp_train(later, first=0, stride=1, update=False, want_grad=True)
+        assert res.pairs == len(rows_t)
+        tgt, w = _targets(now, q, perm, slots, pkg.scenes.dam10k())
+        L, g, _ = ref.loss_and_grad(params.astype(np.float64), f, rows_t, tgt, w)
+        assert res.loss == pytest.approx(L, rel=1e-5)
+        assert np.linalg.norm(grad - g) <= 1e-5 * np.linalg.norm(g)
+        assert sim.coarse_step(1, use_network=True).pairs == len(rows_t)
