@@ -574,6 +574,14 @@ int ensure_mlp_base(sph_ctx* c)
         dalloc(&w.pairs, 1) != hipSuccess ||
         dalloc((char**)&w.sums, kTrainSumsBytes * (kMaxTrainWaves + 1u)) != hipSuccess) {
         (void)hipGetLastError();
+        // All or none: w.params says that the whole group is there.
+        void* got[] = {w.params, w.adam_m, w.adam_v, w.grad, w.pack_a, w.pack_c, w.pairs, w.sums};
+        for (void* p : got)
+            if (p) (void)hipFree(p);
+        w.params = w.adam_m = w.adam_v = w.grad = w.pack_c = nullptr;
+        w.pack_a = nullptr;
+        w.pairs = nullptr;
+        w.sums = nullptr;
         return fail(c, SPH_ERR_NOMEM, "cannot allocate network parameters");
     }
     SPH_HIP(c, hipMemsetAsync(w.adam_m, 0, sizeof(float) * kMlpParams, c->stream));

@@ -94,7 +94,7 @@ constexpr int kMlpPackA = 4 * 64 * 8 + 4 * 2 * 64 * 8 + 2 * 64 * 8;  // 16-bit e
 constexpr int kMlpPackC = 2 * kMlpHidden + 8;                        // float entries
 // Totals of a training step: loss sum, pairs, targets of weight 1.
 constexpr size_t kTrainSumsBytes = 24;
-constexpr uint32_t kMaxTrainWaves = 4u * 2048u;
+constexpr uint32_t kMaxTrainWaves = 4u * 2048u;  // waves of the forward pass, 4 a workgroup
 
 // Each launcher enqueues one kernel on `s` and returns hipGetLastError().
 hipError_t launch_set_scene(hipStream_t s, SceneDev* dst, const SceneDev& value);
