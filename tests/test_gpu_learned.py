@@ -15,7 +15,6 @@ import os
 
 import numpy as np
 import pytest
-import scipy.spatial
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -88,6 +87,15 @@ def _targets(state_now, state_later, perm, slots, sc):
         ok &= np.all(np.isfinite(ps), axis=1) & np.all((np.abs(ps - lo) > 1e-6) & (np.abs(ps - hi) > 1e-6), axis=1)
     tgt = np.where(ok[:, None], acc / NORM["acc_scale"], 0.0)
     return tgt, ok.astype(np.float64)
+
+
+def _cluster(orc, n, seed=3):
+    """n particles, each within h of every other."""
+    rng = np.random.default_rng(seed)
+    p = orc.particles(n)
+    p["pos"][:, :3] = rng.uniform(0.0, 0.008, (n, 3)).astype(np.float32)
+    p["vel"][:, :3] = rng.normal(0, 5, (n, 3)).astype(np.float32)
+    return p
 
 
 def test_training_gradient_matches_fp64(pkg, orc, ref, gpu_lib):
@@ -214,6 +222,7 @@ def test_predict_mfma_matches_fp32(pkg, orc, ref, gpu_lib):
     params[ref.NPARAMS - 195:] += np.random.default_rng(20).normal(0, 0.05, 195).astype(np.float32)
     sim.mlp_set(params, _norm(pkg))
     p32 = sim.mlp_predict(path=0)
+    _poison_predictions(sim, pkg, ref, params)
     pbf = sim.mlp_predict(path=1)
     assert np.all(np.isfinite(pbf))
     rel = np.linalg.norm(pbf - p32) / np.linalg.norm(p32)
@@ -226,6 +235,7 @@ def test_predict_mfma_matches_fp32(pkg, orc, ref, gpu_lib):
         dense.upload(p)
         dense.mlp_set(params, _norm(pkg))
         a = dense.mlp_predict(path=0)
+        _poison_predictions(dense, pkg, ref, params)
         b = dense.mlp_predict(path=1)
         assert np.linalg.norm(b - a) / np.linalg.norm(a) < 2e-2
 
@@ -242,6 +252,7 @@ def test_predict_mfma_every_stencil_size(pkg, orc, ref, gpu_lib, sub):
     p2 = sim.mlp_predict(path=1)
     sim.set_tuning(cells_per_h=sub)
     p32 = sim.mlp_predict(path=0)
+    _poison_predictions(sim, pkg, ref, params)
     pbf = sim.mlp_predict(path=1)
     assert np.all(np.isfinite(pbf))
     assert np.linalg.norm(pbf - p32) / np.linalg.norm(p32) < 2e-2
@@ -255,6 +266,7 @@ def test_predict_mfma_every_stencil_size(pkg, orc, ref, gpu_lib, sub):
         dense.set_tuning(cells_per_h=sub)
         dense.mlp_set(params, _norm(pkg))
         a = dense.mlp_predict(path=0)
+        _poison_predictions(dense, pkg, ref, params)
         b = dense.mlp_predict(path=1)
         assert np.linalg.norm(b - a) / np.linalg.norm(a) < 2e-2
 
@@ -399,25 +411,86 @@ def test_dam8m_learned_leg(pkg, orc, gpu_lib):
         assert m.nonfinite <= 2 * mp.nonfinite + 100, (m.nonfinite, mp.nonfinite)
 
 
+def _count_pairs_only(ref, value):
+    """A network whose message is `value` for every pair."""
+    params = np.zeros(ref.NPARAMS, np.float32)
+    params[-3:] = value
+    return params
+
+
+def _poison_predictions(sim, pkg, ref, params):
+    """Leaves 10^6 per neighbour in the prediction buffer, then loads `params`:
+    a target that the next pass leaves out shows."""
+    sim.mlp_set(_count_pairs_only(ref, 1e6), _norm(pkg))
+    sim.mlp_predict(path=0)
+    sim.mlp_set(params, _norm(pkg))
+
+
+def _assert_gradient_is_the_sum_over(sim, later, k):
+    """The training gradient over all particles is the weighted sum of those of
+    every k-th from 0 .. k-1.  Bound: each is within 1e-6 of its norm or better
+    (float32 sums of some 2,048 rows, added in double)."""
+    res, grad = sim.mlp_train(later, first=0, stride=1, update=False, want_grad=True)
+    parts = [sim.mlp_train(later, first=i, stride=k, update=False, want_grad=True) for i in range(k)]
+    for name in ("pairs", "targets", "weighted"):
+        assert getattr(res, name) == sum(getattr(r, name) for r, _ in parts)
+    assert res.loss * res.weighted == pytest.approx(sum(r.loss * r.weighted for r, _ in parts), rel=1e-9)
+    got = grad.astype(np.float64) * res.weighted
+    want = sum(g.astype(np.float64) * r.weighted for r, g in parts)
+    size = sum(np.linalg.norm(g.astype(np.float64)) * r.weighted for r, g in parts)
+    assert np.linalg.norm(got) > 0.0
+    assert np.linalg.norm(got - want) <= 1e-6 * (np.linalg.norm(got) + size), (np.linalg.norm(got - want), np.linalg.norm(got))
+    return res
+
+
 @pytest.mark.parametrize("n", [513, 65535, 65536, 65601])
 def test_network_takes_every_target_once(pkg, orc, ref, gpu_lib, n):
     """Targets go to the XCDs one a wave below 65,536 and in runs of 64 from
-    there: pairs counted on the device against a k-d tree, between its counts at
-    distances a float32 rounding (1e-6) below and above h."""
+    there, to waves of 4 or (backward pass) 8 a workgroup.  Messages that count a target's
+    pairs, into a buffer that held others, are the same on both paths and add up
+    to the oracle's count, up to pairs that float32 rounding decides; so does what the
+    16-bit pass and the training step count; the gradient is that of two halves,
+    dealt in another way."""
     rng = np.random.default_rng(n)
     side = (n * 1e-6) ** (1.0 / 3.0)
     p = orc.particles(n)
     p["pos"][:, :3] = rng.uniform(0.0, side, (n, 3)).astype(np.float32)
-    with pkg.Simulation(n, boundaries=pkg.sph.make_boundary((0.0,) * 3, (side,) * 3)) as sim, pkg.Simulation(n) as later:
+    q = p.copy()
+    q["vel"][:, :3] = rng.normal(0, 5, (n, 3)).astype(np.float32)
+    bounds = (0.0,) * 3, (side,) * 3
+    want, unsure = orc.count_pairs(orc.pos64(p), b=orc.make_boundary(*bounds))
+    with pkg.Simulation(n, boundaries=pkg.sph.make_boundary(*bounds)) as sim, pkg.Simulation(n) as later:
         sim.upload(p)
-        later.upload(p)
+        later.upload(q)
+        counts = []
+        for path in (1, 0):
+            _poison_predictions(sim, pkg, ref, _count_pairs_only(ref, 1.0))
+            counts.append(sim.mlp_predict(path=path))
+        assert np.array_equal(counts[0], counts[1])
+        assert abs(counts[0][:, 0].astype(np.float64).sum() - want) <= unsure
         sim.mlp_set(ref.init_params(3), _norm(pkg))
-        assert np.isfinite(sim.mlp_predict(path=1)).all()
-        res, _ = sim.mlp_train(later, first=0, stride=1, update=False, want_grad=True)
-        tree = scipy.spatial.cKDTree(p["pos"][:, :3].astype(np.float64))
-        h = float(orc.smoothing_length())
-        low, high = (tree.count_neighbors(tree, h * f) - n for f in (1 - 1e-6, 1 + 1e-6))
-        assert low <= res.pairs <= high and res.targets == n
+        res = _assert_gradient_is_the_sum_over(sim, later, 2)
+        assert abs(res.pairs - want) <= unsure and res.targets == n
+        assert sim.coarse_step(1, use_network=True).pairs == res.pairs
+
+
+def test_training_gradient_over_several_targets_a_wave(pkg, orc, ref, gpu_lib):
+    """6,144 targets of 1,535 neighbours, three to each wave of the backward
+    pass: a wave moves its sums to its partial after two of them (more than
+    2,048 rows) and once more at the end.  Every third and every fourth target
+    alone give a wave one at most."""
+    n, m = 1536, 4
+    p = np.concatenate([_cluster(orc, n, seed) for seed in range(m)])
+    p["pos"][:, 0] += np.repeat(0.1 * np.arange(m, dtype=np.float32), n)
+    q = p.copy()
+    q["vel"][:, :3] += np.random.default_rng(5).normal(0, 5, (n * m, 3)).astype(np.float32)
+    with pkg.Simulation(n * m) as sim, pkg.Simulation(n * m) as later:
+        sim.upload(p)
+        later.upload(q)
+        sim.mlp_set(ref.init_params(3), _norm(pkg))
+        for k in (3, 4):
+            res = _assert_gradient_is_the_sum_over(sim, later, k)
+            assert res.pairs == m * n * (n - 1) and res.targets == m * n
 
 
 @pytest.mark.parametrize("n", [1, 2, 16, 17, 18, 130, 193, 700])
@@ -474,15 +547,6 @@ def test_network_tiles(pkg, orc, ref, gpu_lib, n, sub):
             L, g, _ = ref.loss_and_grad(params.astype(np.float64), f, rows_t, tgt, w)
             assert res.loss == pytest.approx(L, rel=1e-5)
             assert np.linalg.norm(grad - g) <= 1e-5 * np.linalg.norm(g)
-
-
-def _cluster(orc, n, seed=3):
-    """n particles, each within h of every other."""
-    rng = np.random.default_rng(seed)
-    p = orc.particles(n)
-    p["pos"][:, :3] = rng.uniform(0.0, 0.008, (n, 3)).astype(np.float32)
-    p["vel"][:, :3] = rng.normal(0, 5, (n, 3)).astype(np.float32)
-    return p
 
 
 def test_messages_16bit_keep_first_layer_weights(pkg, orc, ref, gpu_lib):
