@@ -106,7 +106,7 @@ hipError_t launch_lattice(hipStream_t s, sph_particle_t* aos, uint32_t first, co
 hipError_t launch_clear_counts(hipStream_t s, uint32_t* count, uint32_t ncount, uint32_t* bsum, uint32_t nbsum);
 hipError_t launch_refresh_extras(hipStream_t s, const DeviceState& d);
 // Counts B into its cells; from_aos copies the AoS pos/vel into B first.
-// block_sums counts the scan's block sums too (slots in near cell order only).
+// block_sums counts the scan's block sums too (a small state in near cell order only).
 hipError_t launch_hash_count(hipStream_t s, const DeviceState& d, bool from_aos, bool block_sums);
 hipError_t launch_scan_reduce(hipStream_t s, const DeviceState& d);
 hipError_t launch_scan_top(hipStream_t s, const DeviceState& d);

@@ -193,7 +193,9 @@ __device__ __forceinline__ void count_into_cell(uint32_t k, bool active, uint32_
     if (active) slot[s] = base + (uint32_t)(lane - my_head);
     // With bsum, the scan's block sums (kScanBlock cells each) are counted
     // alongside, so the build needs no reduction pass over the cells.  Worth it
-    // only for cell-sorted slots, where a wave's keys fall in one or two blocks.
+    // only for cell-sorted slots, where a wave's keys fall in one or two blocks,
+    // and where not too many waves count at once (the fused step's are spread
+    // over its force work).
     if (!bsum) return;
     const uint32_t bk = k / (uint32_t)kScanBlock;
     const uint32_t bprev = __shfl_up(bk, 1u);
@@ -207,8 +209,8 @@ __device__ __forceinline__ void count_into_cell(uint32_t k, bool active, uint32_
 // also counts the scan's block sums, so a step that follows one starts its
 // build at the scan.  With FROM_AOS it first copies the AoS positions and
 // velocities into B through perm (one pass and one launch instead of two: 25
-// against 38 us at 1M particles).  bsum is null where B may be in any order
-// (after an upload), where per-particle block-sum atomics would contend;
+// against 38 us at 1M particles).  bsum is null where block-sum
+// atomics would contend, in a large state or one in any order (after an upload);
 // k_scan_reduce then sums them.
 template <bool FROM_AOS>
 __global__ __launch_bounds__(kTile) void k_hash_count(const Tile* __restrict__ tiles, const SceneDev* __restrict__ scenes,

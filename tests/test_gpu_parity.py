@@ -462,3 +462,21 @@ def test_pass_loop_counts_with_block_sums(pkg, orc, gpu_lib):
             sim.upload(sim.download()[:100])
             advance(2)
         assert passes.download().tobytes() == fused.download().tobytes()
+
+
+@pytest.mark.parametrize("n", [16384, 16385, 60000])
+def test_pass_loop_on_both_sides_of_the_block_sum_limit(pkg, orc, gpu_lib, n):
+    """Loops of passes count the scan's block sums with the cells up to 16,384
+    particles and by the reduction above.  Same bits as fused steps."""
+    sc = pkg.scenes.dam1m()
+    p = orc.lattice(sc.nx, sc.ny, sc.nz, sc.spacing, sc.origin, sc.jitter, sc.seed, count=sc.count)[:n].copy()
+    b = pkg.sph.make_boundary(sc.lower, sc.upper)
+    with pkg.Simulation(n, boundaries=b) as passes, pkg.Simulation(n, boundaries=b) as fused:
+        passes.upload(p)
+        fused.upload(p)
+        for _ in range(4):
+            passes.rho_pres()
+            passes.force()
+            passes.integrate()
+        fused.step(4)
+        assert passes.download().tobytes() == fused.download().tobytes()
