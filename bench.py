@@ -68,7 +68,8 @@ TIMED_REPS = 5
 # beside the plain steps they stand in for.
 LEARNED_WINDOW = 10
 # Learned message pass: flops of the pair MLP 9 -> 64 -> 64 -> 3 per neighbour
-# pair (multiply-adds counted as 2), against MI355X's dense BF16 MFMA peak.
+# pair (multiply-adds counted as 2), against MI355X's dense 16-bit MFMA peak
+# (BF16 and FP16 alike).
 MLP_FLOPS_PER_PAIR = 2 * (9 * 64 + 64 * 64 + 64 * 3)
 # Neighbour build (no reference counterpart), compulsory bytes per particle of
 # the kernels each step launches (the cell key and count of every particle are
@@ -214,8 +215,8 @@ def learned_form(pkg, scenes, state, first_step, fine_steps, plain_ms_per_step, 
                 "unit": "TFLOP/s", "frac": tflops / BF16_DENSE_TFLOPS, "launch_ms": msg_ms,
                 "pairs_per_launch": int(mst.pairs), "flops_per_pair": MLP_FLOPS_PER_PAIR,
                 "ps_per_pair": msg_ms * 1e9 / mst.pairs,
-                "binding_roof": "VALU issue: 128 GELU evaluations per pair run on the vector ALUs between the "
-                                "MFMA layers"}
+                "binding_roof": "VALU issue: 128 GELUs per pair lie between the MFMA layers, half as packed FP16 "
+                                "polynomials, half as LDS lookups with vector address work"}
     # The same window from the same state for both forms: LEARNED_WINDOW coarse
     # steps of the network alone (no judge) and the 4x as many plain steps
     # they stand in for.

@@ -335,8 +335,9 @@ int sph_mlp_train(sph_ctx* ctx, const sph_ctx* later, const sph_train_opts_t* op
                   sph_train_result_t* result);
 
 /* Summed messages of every particle at the current state (AoS order, 3 floats
- * per particle, units of acc_scale).  path 0: float32 kernel; 1: BF16 MFMA
- * kernel.  Runs the density pass first (as sph_rho_pres). */
+ * per particle, units of acc_scale).  path 0: float32 kernel; 1: 16-bit MFMA
+ * kernel (BF16 inputs, FP16 activations, float32 sums).  Runs the density pass
+ * first (as sph_rho_pres). */
 int sph_mlp_predict(sph_ctx* ctx, int path, float* out);
 
 /* n coarse steps (each = 4 fine steps of simulated time), with the plain
